@@ -397,7 +397,12 @@ static void dispatch_class(int dim, int mat, int bucket, F &&f) {
 // Sorts every member; the sorted planes stay in the workspaces (descs_src).
 static int group_sort(aq_group *g, hipStream_t st) {
   const int32_t n = (int32_t)g->sims.size();
-  for (const GroupClass &f : g->classes)
+  LAUNCH_CHECK();
+  for (aq_sim *s : g->sims) {
+    const int rc = sort_begin(s, st);
+    if (rc) return rc;
+  }
+  for (const GroupClass &f : g->classes) {
     dispatch_class(f.dim, f.mat, f.bucket, [&](auto tag_) {
       TAG_TYPES(tag_)
       (void)MAT;
@@ -405,8 +410,11 @@ static int group_sort(aq_group *g, hipStream_t st) {
       hipLaunchKernelGGL((k_group_keys<DIM, NW32>), dim3(f.keys_blocks), dim3(256), 0, st,
                          (const GroupSortArgs *)(g->sorts + f.sort0), (const int32_t *)f.keys_prefix, f.nsims);
     });
+    LAUNCH_CHECK();
+  }
   hipLaunchKernelGGL(k_group_counts, dim3(g->counts_blocks), dim3(kCountThreads), 0, st,
                      (const GroupSortArgs *)g->sorts, (const int32_t *)g->counts_prefix, n);
+  LAUNCH_CHECK();
   for (const GroupGather &q : g->gathers) {
     if (q.dim == 3)
       hipLaunchKernelGGL(k_group_scan<3>, dim3(q.scan_blocks), dim3(256), 0, st, (const GroupSortArgs *)q.sorts,
@@ -414,11 +422,15 @@ static int group_sort(aq_group *g, hipStream_t st) {
     else
       hipLaunchKernelGGL(k_group_scan<2>, dim3(q.scan_blocks), dim3(256), 0, st, (const GroupSortArgs *)q.sorts,
                          (const int32_t *)q.scan_prefix, q.nsims);
+    LAUNCH_CHECK();
   }
   hipLaunchKernelGGL(k_group_scatter, dim3(g->scatter_blocks), dim3(256), 0, st, (const GroupSortArgs *)g->sorts,
                      (const int32_t *)g->scatter_prefix, n);
+  LAUNCH_CHECK();
   hipLaunchKernelGGL(k_group_finish, dim3(g->finish_blocks), dim3(256), 0, st, (const GroupSortArgs *)g->sorts,
                      (const int32_t *)g->finish_prefix, n);
+  LAUNCH_CHECK();
+  for (aq_sim *s : g->sims) s->sort_open = false;
   ItemPrefixArgs C{};
   for (size_t c = 0; c < g->classes.size(); ++c) {
     C.descs[c] = g->classes[c].descs;

@@ -423,6 +423,12 @@ __global__ void k_fill_u32(uint32_t *a, uint32_t v, int64_t n) {
   if (i < n) a[i] = v;
 }
 
+int fill_u32(uint32_t *a, uint32_t v, int64_t n, hipStream_t st) {
+  hipLaunchKernelGGL(k_fill_u32, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, a, v, n);
+  LAUNCH_CHECK();
+  return AQ_OK;
+}
+
 // ---- reductions ----------------------------------------------------------------
 // Per-component max / min of the state: grid-stride blocks fold their
 // largest values and largest negated values into their slots of part

@@ -117,6 +117,7 @@ struct aq_sim {
   // sorted copy in the workspace, until a G2P writes every particle back
   // (never set between API calls)
   const void *src = nullptr;
+  bool sort_open = false;  // a sort failed between its launches: its cell counters and marks may not be zero
   bool dither_any;
   bool stream_order;  // the encoder's field order has non-decreasing offsets
   int64_t ws_bytes;
@@ -250,10 +251,17 @@ ColliderK collider_at(const aq_sim *s, uint32_t step);
 // takes parity 0 (every call leaves this state, so that a captured call
 // replays on the state it was recorded from).
 int settle_list(aq_sim *s, hipStream_t st);
+int fill_u32(uint32_t *a, uint32_t v, int64_t n, hipStream_t st);
 // aq_sort.hip: sort of `state`; defer: the sorted planes stay in the
 // workspace (s->src), for a P2G and then a G2P of every particle that writes
 // them to `state` (saves the copy back: a read and a write of every record)
 int launch_sort(aq_sim *s, void *state, int64_t n, int32_t *ids, bool defer, hipStream_t st);
+// Around a sort's launches (of this simulation alone or of a group): begin
+// clears what a failed sort left in the counters and drops the items, whose
+// tables the launches overwrite; end notes the new order (src: planes of the
+// sorted copy, or null).
+int sort_begin(aq_sim *s, hipStream_t st);
+void sort_end(aq_sim *s, const void *state, int64_t n, const void *src);
 struct SortBuf;
 SortBuf sort_buf(const aq_sim *s, void *state, int64_t n, int32_t *ids);
 unsigned sort_finish_blocks(const SortBuf &b);

@@ -70,8 +70,34 @@ unsigned sort_finish_blocks(const SortBuf &b) {
   return (unsigned)(p > m ? p : m);
 }
 
+int sort_begin(aq_sim *s, hipStream_t st) {
+  int rc;
+  if (s->sort_open) {
+    if ((rc = fill_u32(s->ccount, 0u, s->nodes, st))) return rc;
+    if ((rc = fill_u32(s->marks, 0u, s->nblocks, st))) return rc;
+  }
+  s->sort_open = true;
+  s->have_items = false;
+  return AQ_OK;
+}
+
+void sort_end(aq_sim *s, const void *state, int64_t n, const void *src) {
+  s->sort_open = false;
+  s->commit_pending = 0;
+  s->list_parity = 0;
+  s->have_items = true;
+  s->items_state = state;
+  s->items_n = n;
+  s->src = src;
+}
+
+// Every launch is checked before the next: the scatter indexes with what the
+// kernels before it wrote.
 int launch_sort(aq_sim *s, void *state, int64_t n, int32_t *ids, bool defer, hipStream_t st) {
   if (n == 0) return AQ_OK;
+  LAUNCH_CHECK();  // an error that was there before is reported with nothing launched
+  const int rc = sort_begin(s, st);
+  if (rc) return rc;
   const StateK sk = make_state(s, state, nullptr);
   const CodecK cod = make_codec(s, 0u);
   const SortBuf b = sort_buf(s, state, n, ids);
@@ -81,6 +107,7 @@ int launch_sort(aq_sim *s, void *state, int64_t n, int32_t *ids, bool defer, hip
     hipLaunchKernelGGL((k_sort_keys<DIM, ST, NW32, T>), dim3(pblocks(n)), dim3(256), 0, st, sk, cod, params_of<T>(s),
                        b);
   });
+  LAUNCH_CHECK();
   const bool d3 = s->d.dim == 3;
   if (b.m <= kScanInline) {
     if (d3)
@@ -90,27 +117,28 @@ int launch_sort(aq_sim *s, void *state, int64_t n, int32_t *ids, bool defer, hip
   } else {
     const unsigned g = (unsigned)((b.m + 255) / 256);
     hipLaunchKernelGGL(k_sort_counts, dim3((unsigned)((b.m + 63) / 64)), dim3(kCountThreads), 0, st, b);
+    LAUNCH_CHECK();
     if (d3)
       hipLaunchKernelGGL(k_sort_scan<3>, dim3(g), dim3(256), 0, st, b);
     else
       hipLaunchKernelGGL(k_sort_scan<2>, dim3(g), dim3(256), 0, st, b);
   }
-  const unsigned f = sort_finish_blocks(b);
-  if (s->d.storage == AQ_STORE_F32) {
-    hipLaunchKernelGGL(k_sort_scatter<uint32_t>, dim3(pblocks(n)), dim3(256), 0, st, b);
-    if (!defer) hipLaunchKernelGGL((k_sort_finish<uint32_t, true>), dim3(f), dim3(256), 0, st, b);
-  } else {
-    hipLaunchKernelGGL(k_sort_scatter<uint64_t>, dim3(pblocks(n)), dim3(256), 0, st, b);
-    if (!defer) hipLaunchKernelGGL((k_sort_finish<uint64_t, true>), dim3(f), dim3(256), 0, st, b);
-  }
-  if (defer) hipLaunchKernelGGL((k_sort_finish<uint32_t, false>), dim3(f), dim3(256), 0, st, b);
   LAUNCH_CHECK();
-  s->commit_pending = 0;
-  s->list_parity = 0;
-  s->have_items = true;
-  s->items_state = state;
-  s->items_n = n;
-  s->src = defer ? s->tmp_state : nullptr;
+  const bool words = s->d.storage != AQ_STORE_F32;  // planes of 8 bytes
+  if (words)
+    hipLaunchKernelGGL(k_sort_scatter<uint64_t>, dim3(pblocks(n)), dim3(256), 0, st, b);
+  else
+    hipLaunchKernelGGL(k_sort_scatter<uint32_t>, dim3(pblocks(n)), dim3(256), 0, st, b);
+  LAUNCH_CHECK();
+  const unsigned f = sort_finish_blocks(b);
+  if (defer)
+    hipLaunchKernelGGL((k_sort_finish<uint32_t, false>), dim3(f), dim3(256), 0, st, b);
+  else if (words)
+    hipLaunchKernelGGL((k_sort_finish<uint64_t, true>), dim3(f), dim3(256), 0, st, b);
+  else
+    hipLaunchKernelGGL((k_sort_finish<uint32_t, true>), dim3(f), dim3(256), 0, st, b);
+  LAUNCH_CHECK();
+  sort_end(s, state, n, defer ? s->tmp_state : nullptr);
   return AQ_OK;
 }
 
