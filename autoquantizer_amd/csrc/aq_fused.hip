@@ -12,7 +12,6 @@ int launch_g2p2g(aq_sim *s, void *state, int64_t n, const int32_t *ids, uint32_t
   if (n == 0) return AQ_OK;
   StateK sk = make_state(s, state, ids);
   CodecK cod = make_codec(s, step);
-  s->src = nullptr;  // every particle is written to `state`
   if (*tiled && s->jit_fn) {
     ParamsT<float> P = s->pf;
     const int4 *items = s->items;
@@ -26,6 +25,7 @@ int launch_g2p2g(aq_sim *s, void *state, int64_t n, const int32_t *ids, uint32_t
     uint32_t ctl = take_list_ctl(s);
     void *args[] = {&sk, &cod, &P, &n, &items, &nitems, &gv, &tl, &gf, &ff, &fl, &gc, &ctl, &bm};
     HIP_TRY(hipModuleLaunchKernel(s->jit_fn, tblocks(s, n), 1, 1, kItem, 1, 1, 0, st, args, nullptr));
+    s->src = nullptr;  // every particle is written to `state`
     return AQ_OK;
   }
   uint32_t *bm = s->bmargin + (int64_t)s->list_parity * s->nblocks;  // the next gather's flags
@@ -51,5 +51,6 @@ int launch_g2p2g(aq_sim *s, void *state, int64_t n, const int32_t *ids, uint32_t
                          params_of<T>(s), n, (const vec4_t<T> *)s->grid_v, (vec4_t<T> *)s->grid_f, s->fflags);
   });
   LAUNCH_CHECK();
+  s->src = nullptr;
   return AQ_OK;
 }

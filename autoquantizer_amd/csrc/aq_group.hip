@@ -164,6 +164,7 @@ struct aq_group {
   std::vector<GroupClass> classes;
   std::vector<GroupGather> gathers;
   // all members, class after class
+  std::vector<int> order;
   GroupSortArgs *sorts;
   int32_t *counts_prefix, *scatter_prefix, *finish_prefix;
   int32_t counts_blocks, scatter_blocks, finish_blocks;
@@ -307,7 +308,7 @@ extern "C" int aq_group_create(aq_sim *const *sims, void *const *states, const i
     return a;
   };
   const auto particles = [&](int i) { return (g->ns[i] + 255) / 256; };
-  std::vector<int> all;
+  std::vector<int> &all = g->order;
   for (size_t c = 0; c < g->classes.size(); ++c) {
     GroupClass &f = g->classes[c];
     f.nsims = (int32_t)cmem[c].size();
@@ -397,7 +398,6 @@ static void dispatch_class(int dim, int mat, int bucket, F &&f) {
 // Sorts every member; the sorted planes stay in the workspaces (descs_src).
 static int group_sort(aq_group *g, hipStream_t st) {
   const int32_t n = (int32_t)g->sims.size();
-  LAUNCH_CHECK();
   for (aq_sim *s : g->sims) {
     const int rc = sort_begin(s, st);
     if (rc) return rc;
@@ -430,7 +430,7 @@ static int group_sort(aq_group *g, hipStream_t st) {
   hipLaunchKernelGGL(k_group_finish, dim3(g->finish_blocks), dim3(256), 0, st, (const GroupSortArgs *)g->sorts,
                      (const int32_t *)g->finish_prefix, n);
   LAUNCH_CHECK();
-  for (aq_sim *s : g->sims) s->sort_open = false;
+  for (int32_t i = 0; i < n; ++i) sort_end(g->sims[i], g->states[i], g->ns[i], g->sims[i]->tmp_state);
   ItemPrefixArgs C{};
   for (size_t c = 0; c < g->classes.size(); ++c) {
     C.descs[c] = g->classes[c].descs;
@@ -474,8 +474,10 @@ static int group_tiled(aq_group *g, uint32_t step, int workgroups, bool src, int
                          (const TiledArgs<float> *)(src ? f.descs_src : f.descs), (const int32_t *)f.prefix, f.nsims,
                          step, parity, masked ? 1 : 0, commit);
     });
+    LAUNCH_CHECK();
+    if (DO_G2P)  // every particle of the class is written to its caller's planes
+      for (int32_t k = 0; k < f.nsims; ++k) g->sims[g->order[f.sort0 + k]]->src = nullptr;
   }
-  LAUNCH_CHECK();
   return AQ_OK;
 }
 
@@ -514,15 +516,10 @@ extern "C" int aq_group_advance(aq_group *g, int nsteps, uint32_t step0, int sor
   if (workgroups < 0 || workgroups > 8192 || workgroups % 8 != 0)
     return fail(AQ_ERR_INVALID, "workgroups must be a multiple of 8 in [0, 8192]");
   if (nsteps == 0) return AQ_OK;
+  LAUNCH_CHECK();  // an error that was there before is reported with nothing launched
   const int rc = group_run(g, nsteps, step0, sort_every, workgroups, (hipStream_t)stream);
-  for (size_t i = 0; i < g->sims.size(); ++i) {
-    aq_sim *s = g->sims[i];
-    s->src = nullptr;
-    s->commit_pending = 0;
-    s->list_parity = 0;
-    s->have_items = rc == AQ_OK;  // the items of the last sort describe the members' states
-    s->items_state = g->states[i];
-    s->items_n = g->ns[i];
-  }
+  // the lists are left as every call leaves them (settle_list), the items of the last sort describe the states
+  if (rc)
+    for (aq_sim *s : g->sims) drop_run(s, (hipStream_t)stream);
   return rc;
 }

@@ -1281,11 +1281,9 @@ static int advance_impl(aq_sim *s, void *state, int64_t n, int nsteps, uint32_t 
   if (rc) return rc;
   if (nsteps < 0) return fail(AQ_ERR_INVALID, "negative step count");
   if (nsteps == 0 || n == 0) return AQ_OK;
+  LAUNCH_CHECK();  // an error that was there before is reported with nothing launched
   rc = advance_run(s, state, n, nsteps, step0, sort_every, ids, st, tm, mxmn);
-  if (rc && s->src) {  // a failed launch left the sorted planes in the workspace: the items do not describe `state`
-    s->src = nullptr;
-    s->have_items = false;
-  }
+  if (rc) drop_run(s, st);
   return rc;
 }
 

@@ -48,7 +48,6 @@ int launch_g2p(aq_sim *s, void *state, int64_t n, const int32_t *ids, uint32_t s
   CodecK cod = make_codec(s, step);
   const bool tiled = items_valid(s, state, n);
   uint32_t ctl = tiled ? take_list_ctl(s) : 0u;  // G2P only: carries a commit, appends nothing
-  s->src = nullptr;  // every particle is written to `state`
   uint32_t *bm = nullptr;
   if (tiled && s->list_parity == 1) {  // the masks of parity 0 cleared (settle_list)
     bm = s->bmargin;
@@ -65,6 +64,7 @@ int launch_g2p(aq_sim *s, void *state, int64_t n, const int32_t *ids, uint32_t s
     uint32_t *gc = s->gcnt;
     void *args[] = {&sk, &cod, &P, &n, &items, &nitems, &gv, &tl, &gf, &ff, &fl, &gc, &ctl, &bm};
     HIP_TRY(hipModuleLaunchKernel(s->jit_fn_g2p, tblocks(s, n), 1, 1, kItem, 1, 1, 0, st, args, nullptr));
+    s->src = nullptr;  // every particle is written to `state`
     return AQ_OK;
   }
   dispatch(s, [&](auto tag_) {
@@ -89,6 +89,7 @@ int launch_g2p(aq_sim *s, void *state, int64_t n, const int32_t *ids, uint32_t s
                          params_of<T>(s), n, (const vec4_t<T> *)s->grid_v);
   });
   LAUNCH_CHECK();
+  s->src = nullptr;
   return AQ_OK;
 }
 

@@ -262,6 +262,9 @@ int launch_sort(aq_sim *s, void *state, int64_t n, int32_t *ids, bool defer, hip
 // sorted copy, or null).
 int sort_begin(aq_sim *s, hipStream_t st);
 void sort_end(aq_sim *s, const void *state, int64_t n, const void *src);
+// After a run that failed: planes that no G2P wrote back are copied to the
+// caller's (whose ids have the new order already), the items are dropped.
+void drop_run(aq_sim *s, hipStream_t st);
 struct SortBuf;
 SortBuf sort_buf(const aq_sim *s, void *state, int64_t n, int32_t *ids);
 unsigned sort_finish_blocks(const SortBuf &b);

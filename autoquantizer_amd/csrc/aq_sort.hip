@@ -91,11 +91,25 @@ void sort_end(aq_sim *s, const void *state, int64_t n, const void *src) {
   s->src = src;
 }
 
+void drop_run(aq_sim *s, hipStream_t st) {
+  if (s->src) {
+    const size_t esz = s->d.storage == AQ_STORE_F32 ? 4 : 8;
+    const size_t pitch = (size_t)s->d.capacity * esz;
+    const size_t planes = (size_t)(s->d.storage == AQ_STORE_QUANT ? s->d.nwords : s->d.ncomp);
+    (void)hipMemcpy2DAsync((void *)s->items_state, pitch, s->src, pitch, (size_t)s->items_n * esz, planes,
+                           hipMemcpyDeviceToDevice, st);
+    s->src = nullptr;
+  }
+  s->have_items = false;
+  s->commit_pending = 0;  // of lists that the next sort makes anew
+  s->list_parity = 0;
+  (void)hipGetLastError();  // the run's error is reported by its caller, once
+}
+
 // Every launch is checked before the next: the scatter indexes with what the
 // kernels before it wrote.
 int launch_sort(aq_sim *s, void *state, int64_t n, int32_t *ids, bool defer, hipStream_t st) {
   if (n == 0) return AQ_OK;
-  LAUNCH_CHECK();  // an error that was there before is reported with nothing launched
   const int rc = sort_begin(s, st);
   if (rc) return rc;
   const StateK sk = make_state(s, state, nullptr);
@@ -145,5 +159,6 @@ int launch_sort(aq_sim *s, void *state, int64_t n, int32_t *ids, bool defer, hip
 extern "C" int aq_sort(aq_sim *s, void *state, int64_t n, int32_t *ids, void *stream) {
   const int rc = check_n(s, state, n);
   if (rc) return rc;
+  LAUNCH_CHECK();  // an error that was there before is reported with nothing launched
   return launch_sort(s, state, n, ids, false, (hipStream_t)stream);
 }

@@ -3,8 +3,9 @@ HIP runtime (compiled here with gcc) that records every launch and copy and
 lets a chosen launch fail, for every launch of a run in turn.
 
 After a failed launch a sort must not go on (its later kernels would index
-with tables that were not written), and the next sort must clear what the
-failed one left in its counters.
+with tables that were not written), the next sort must clear what the failed
+one left in its counters, the caller's planes and ids must be in the same
+order, and the items of the failed run must not be used again.
 """
 import ctypes
 import importlib.util
@@ -148,6 +149,10 @@ def _child(fake):
     F.fake_reset(0, 719)
     out["left"] = {"rc": L.aq_advance(s[0], s[1], s[3], 4, 0, 2, s[2], None), "run": log(),
                    "again": L.aq_advance(s[0], s[1], s[3], 4, 0, 2, s[2], None)}
+    F.fake_reset(0, 719)
+    out["left"]["sorted"] = L.aq_advance(s[0], s[1], s[3], 4, 0, 2, s[2], None)
+    _lib.check(L.aq_p2g(s[0], s[1], s[3], None))
+    out["left"]["p2g"] = log()
     print(json.dumps(out))
 
 
@@ -166,6 +171,7 @@ def logs(tmp_path_factory):
 
 
 SORTS = re.compile(r"k_(sort|group)_(keys|counts|count_scan|scan|scatter|finish)")
+G2P = re.compile(r"k_tiledI.*?fLb1|k_tiled_groupILi\dELi\dELi\d+ELb1")
 
 
 def _split(r):
@@ -201,11 +207,39 @@ def test_failed_sort_stops_and_is_cleared(logs, kind):
             assert first == [open_sort, open_sort], (r["fail"], k, s)
 
 
+@pytest.mark.parametrize("kind", ["advance", "group"])
+def test_failed_run_leaves_planes_and_ids_in_one_order(logs, kind):
+    for r in logs[kind]:
+        if r["rc"] == 0:
+            continue
+        before, failed, after = _split(r)
+        # planes of the last complete sort that no G2P has written back: all of a run's, one class of a group's
+        last = max([i for i, x in enumerate(before) if "finish" in x], default=-1)
+        written = [x for x in before[last + 1:] if G2P.search(x)] if last >= 0 else []
+        classes = {re.search(r"k_tiled_groupI(Li\dELi\dELi\d+)", x).group(1) for x in written if "group" in x}
+        for k, state in enumerate(r["states"]):
+            mine = bool(written) if kind == "advance" else any(c.startswith("Li3" if k == 1 else "Li2") for c in classes)
+            want = last >= 0 and not mine
+            assert (f"copy to {state}" in after) == want, (r["fail"], k, failed, after)
+
+
+@pytest.mark.parametrize("kind", ["advance", "group"])
+def test_failed_run_drops_the_items(logs, kind):
+    for r in logs[kind]:
+        for p in r["p2g"]:
+            if r["rc"] == 0:
+                assert "k_tiled" in p[0]
+            else:
+                assert "k_p2g" in p[0], (r["fail"], p)
+
+
 def test_error_left_by_the_caller(logs):
     """An error that an earlier call of the caller left: reported before
-    anything is launched, and not again."""
-    assert logs["left"]["rc"] < 0 and logs["left"]["run"] == []
-    assert logs["left"]["again"] == 0
+    anything is launched, and not again; the items of an earlier sort stay."""
+    left = logs["left"]
+    assert left["rc"] < 0 and left["run"] == []
+    assert left["again"] == 0
+    assert left["sorted"] < 0 and "k_tiled" in left["p2g"][0]
 
 
 if __name__ == "__main__":
