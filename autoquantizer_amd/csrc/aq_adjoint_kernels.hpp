@@ -718,32 +718,6 @@ __global__ void __launch_bounds__(256) k_adj_p2g(const T *__restrict__ st, T *__
 }
 
 // ---- tiled particle phases ---------------------------------------------------
-// LDS sums of the scattered velocity adjoint: one int64 per axis.  The node
-// adjoints are divided by the node's mass, so nodes that little mass reaches
-// need their own relative precision, as float sums have it: with 30 bits of
-// the item's bound, as the tiled P2G keeps them, single particles' grad x was
-// 1.7e-3 of the root mean square off, with 54 it is 3e-4, as with float
-// atomics.  f32 contributions down to 2^-30 of the bound enter exactly.
-template <class T> struct AdjAcc;
-template <> struct AdjAcc<float> {
-  static constexpr int BITS = 54;
-  // x rounded to an integer, |x| < 2^54: x = hi 2^24 + lo in exact steps
-  __device__ static unsigned long long fix(float x) {
-    const float h = truncf(x * 5.9604644775390625e-8f);  // 2^-24
-    const float l = __builtin_rintf(fmaf(h, -16777216.0f, x));
-    return (unsigned long long)((long long)(int32_t)h * 16777216ll + (long long)(int32_t)l);
-  }
-  __device__ static float unfix(unsigned long long q, int k) {
-    const double d = (double)(int32_t)((long long)q >> 32) * 4294967296.0 + (double)(uint32_t)q;
-    return (float)ldexp(d, -k);
-  }
-};
-template <> struct AdjAcc<double> {
-  static constexpr int BITS = AccOf<double>::BITS;
-  __device__ static unsigned long long fix(double x) { return AccOf<double>::fix(x); }
-  __device__ static double unfix(unsigned long long q, int k) { return AccOf<double>::unfix(q, k); }
-};
-
 // Wavefronts per SIMD that registers are kept for (G2P adjoint, P2G adjoint);
 // 3D f64 keeps one.
 template <int DIM, class T> struct AdjWaves {
@@ -753,11 +727,17 @@ template <int DIM, class T> struct AdjWaves {
 
 // G2P adjoint over work items: the velocity tile staged in LDS is read by
 // every particle, and its velocity adjoints w_n u_n (u_n = vb + 4 inv_dx C_b
-// (off_n - fx)) are summed in an LDS tile in fixed point with per-item,
-// per-axis scales, as the tiled P2G sums momentum (tiled_run): with global
-// float atomics (k_adj_g2p) the 81 (3D) atomics a particle bound the phase.
-// 262,144 particles of a 3D fluid, f32: 1630 -> 32 us; 80,000 of a 2D
-// elastic body, f64: 101 -> 8.5 us.
+// (off_n - fx)) are summed in an LDS tile: with global float atomics
+// (k_adj_g2p) the 81 (3D) atomics a particle bound the phase.
+// The sums are doubles, for f32 adjoints too.  The node adjoints are divided
+// by the node's mass afterwards, so a node that little mass reaches, or that
+// lies next to far larger adjoints, needs a sum that is accurate relative to
+// itself.  In fixed point relative to the item's largest adjoints a
+// contribution of 2^-40 of them keeps 22 of its bits (62-bit sums), and the
+// bound, the scale and the rounding cost more than the f64 atomics: 262,144
+// particles of a 3D fluid, f32: 31 us in fixed point, 27 so (1630 with global
+// atomics), of a 3D elastic body 36 and 30; 80,000 of a 2D elastic body, f64:
+// 7.2 both ways (101).
 template <int DIM, int MAT, class T>
 __global__ void __launch_bounds__(kItem) __attribute__((amdgpu_waves_per_eu(AdjWaves<DIM, T>::G2P)))
 k_adj_g2p_tiled(const T *__restrict__ st, const T *__restrict__ adj_next,
@@ -769,11 +749,9 @@ k_adj_g2p_tiled(const T *__restrict__ st, const T *__restrict__ adj_next,
                                                          uint32_t *__restrict__ fflags, int32_t *flist, uint32_t *gcnt,
                                                          uint32_t ctl, uint32_t *bmargin) {
   using TL = Tile<DIM>;
-  using ACC = AdjAcc<T>;
   constexpr int TS = TL::TS, TN = TL::TN, TE = TL::TE, NW = kItem / 64;
   __shared__ vec4_t<T> tv[TS];
-  __shared__ unsigned long long ts[DIM][TS];
-  __shared__ T bpart[NW][3];
+  __shared__ double ts[DIM][TS];
   __shared__ uint32_t bdrift[NW];
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
   // commit of the last list gather's appends, as tiled_body does
@@ -794,7 +772,7 @@ k_adj_g2p_tiled(const T *__restrict__ st, const T *__restrict__ adj_next,
   share.init(tid, P.nb);
   for (int q = tid; q < TS; q += kItem)
 #pragma unroll
-    for (int a = 0; a < DIM; ++a) ts[a][q] = 0ull;
+    for (int a = 0; a < DIM; ++a) ts[a][q] = 0.0;
   for (; it < hi; it += per) {
     const int4 item = items[it];
     int o[3];
@@ -806,67 +784,40 @@ k_adj_g2p_tiled(const T *__restrict__ st, const T *__restrict__ adj_next,
     if (has) adj_g2p_load<DIM, MAT, T>(st, adj_next, cap, p, x, A);
     share.template copy<T>(item, tid, grid_v, tv);
     AdjStencil<T> S;
-    T B[3] = {(T)0, (T)0, (T)0};
     int rel[3] = {0, 0, 0};
     bool inside = false, drift = false;
     if (has) {
       S = adj_stencil<DIM, T>(x, P);
       A.begin(P, S);
-      T W = (T)1;
-#pragma unroll
-      for (int a = 0; a < DIM; ++a) {
-        W *= tmax<T>(tmax<T>(tabs<T>(S.w[a][0]), S.w[a][1]), tabs<T>(S.w[a][2]));
-        W = S.fx[a] == S.fx[a] ? W : S.fx[a];  // a NaN weight must not vanish in tmax
-      }
       inside = true;
 #pragma unroll
       for (int a = 0; a < DIM; ++a) {
-        T m = tabs<T>(A.c[a]);
-#pragma unroll
-        for (int b = 0; b < DIM; ++b) m += tabs<T>(A.A[a][b]);
-        B[a] = W * m * ((T)1 + (T)1 / (T)1024);
         rel[a] = S.base[a] - o[a];
-        inside = inside && rel[a] >= 0 && rel[a] + 2 < TE && S.fx[a] >= (T)0.5 && S.fx[a] <= (T)1.5;
+        inside = inside && rel[a] >= 0 && rel[a] + 2 < TE;
         drift = drift || rel[a] == 0 || rel[a] == TE - 3;
       }
       drift = drift && inside;
-      if (!inside) B[0] = B[1] = B[2] = (T)0;  // scatters by itself, no share in the item's scales
     }
-#pragma unroll
-    for (int a = 0; a < DIM; ++a) B[a] = wave_sum<T>(B[a]);
     const bool wdrift = __ballot(drift) != 0ull;
-    if (lane == 0) {
-#pragma unroll
-      for (int a = 0; a < DIM; ++a) bpart[wave][a] = B[a];
-      bdrift[wave] = wdrift ? 1u : 0u;
-    }
-    __syncthreads();  // tile staged, bounds complete, the previous item's sums written out
+    if (lane == 0) bdrift[wave] = wdrift ? 1u : 0u;
+    __syncthreads();  // tile staged, the previous item's sums written out
     uint32_t d = 0u;
 #pragma unroll
     for (int w = 0; w < NW; ++w) d |= bdrift[w];
     const int ib = it - item_off[item.x];
     const bool margin = d != 0u || ib >= 31;
     if (margin && tid == 0) atomicOr(bmargin + item.x, 1u << (ib < 31 ? ib : 31));
-    int ks[3] = {0, 0, 0};
-    bool finite = true;
-#pragma unroll
-    for (int a = 0; a < DIM; ++a) {
-      T sum = bpart[0][a];
-#pragma unroll
-      for (int w = 1; w < NW; ++w) sum += bpart[w][a];
-      finite = finite && sum <= (T)1.0e37;
-      ks[a] = ACC::BITS - texp<T>(sum * ((T)1 + (T)1 / (T)1024));
-    }
     if (has) {
       T xo[3], jo[AdjG2P<DIM, MAT, T>::NJF];
-      if (inside && finite) {
+      if (inside) {
         const int q0 = TL::slot(rel[0], rel[1], rel[2]);
         A.sums(
             P, S, [&](const int (&off)[3]) { return tv[q0 + TL::slot(off[0], off[1], off[2])]; },
             [&](const int (&off)[3], T w, const T (&u)[3]) {
               const int q = q0 + TL::slot(off[0], off[1], off[2]);
 #pragma unroll
-              for (int a = 0; a < DIM; ++a) atomicAdd(&ts[a][q], ACC::fix(tldexp<T>(w * u[a], ks[a])));
+              for (int a = 0; a < DIM; ++a)
+                __hip_atomic_fetch_add(&ts[a][q], (double)(w * u[a]), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
             },
             xo, jo);
       } else {
@@ -892,12 +843,12 @@ k_adj_g2p_tiled(const T *__restrict__ st, const T *__restrict__ adj_next,
       const int q = share.slot(r);
       vec4_t<T> val;
       val.z = val.w = (T)0;
-      val.x = ACC::unfix(ts[0][q], ks[0]);
-      val.y = ACC::unfix(ts[1][q], ks[1]);
-      if constexpr (DIM == 3) val.z = ACC::unfix(ts[DIM - 1][q], ks[2]);
+      val.x = (T)ts[0][q];
+      val.y = (T)ts[1][q];
+      if constexpr (DIM == 3) val.z = (T)ts[DIM - 1][q];
       dst[nd] = val;
 #pragma unroll
-      for (int a = 0; a < DIM; ++a) ts[a][q] = 0ull;
+      for (int a = 0; a < DIM; ++a) ts[a][q] = 0.0;
     }
     // the next item's copy writes tv only after every thread passed the
     // barrier above (its last reads of tv), and its sums start after the
