@@ -590,7 +590,7 @@ static int32_t max_items_of(const aq_sim_desc *d) {
 static int64_t tile_slots(const aq_sim_desc *d) { return d->dim == 3 ? Tile<3>::STRIDE : Tile<2>::STRIDE; }
 
 enum {
-  WS_GRID_V, WS_GRID_F, WS_FLAGS, WS_GLIST, WS_CCOUNT, WS_MARKS, WS_KEY, WS_RANK, WS_COUNT, WS_OFF, WS_PART, WS_TMP_STATE, WS_TMP_IDS,
+  WS_GRID_V, WS_GRID_F, WS_FLAGS, WS_GLIST, WS_CCOUNT, WS_MARKS, WS_TOP, WS_KEY, WS_RANK, WS_COUNT, WS_OFF, WS_PART, WS_TMP_STATE, WS_TMP_IDS,
   WS_ITEMS, WS_ITEM_OFF, WS_NEAR, WS_TILES, WS_LIMITS, WS_LAYOUT, WS_N
 };
 
@@ -612,6 +612,7 @@ static void ws_plan(const aq_sim_desc *d, int64_t *offs /*[WS_N]*/, int64_t *tot
   sz[WS_COUNT] = (nblocks + 1) * 4;
   sz[WS_CCOUNT] = nodes * 4;  // particles per cell (64 cells per block)
   sz[WS_MARKS] = nblocks * 4;  // blocks with particles
+  sz[WS_TOP] = (chunks + kTop - 1) / kTop * 8;
   sz[WS_OFF] = (nblocks + 1) * 4;
   sz[WS_PART] = chunks * 8;
   sz[WS_TMP_STATE] = state_bytes;
@@ -714,6 +715,7 @@ extern "C" int aq_sim_create(const aq_sim_desc *d, void *ws, int64_t ws_bytes, a
   s->scount = (uint32_t *)(base + offs[WS_COUNT]);
   s->ccount = (uint32_t *)(base + offs[WS_CCOUNT]);
   s->marks = (uint32_t *)(base + offs[WS_MARKS]);
+  s->stop = (uint32_t *)(base + offs[WS_TOP]);
   s->soff = (uint32_t *)(base + offs[WS_OFF]);
   s->spart = (uint32_t *)(base + offs[WS_PART]);
   s->tmp_state = base + offs[WS_TMP_STATE];

@@ -101,7 +101,7 @@ struct aq_sim {
   int32_t list_parity = 0;     // parity of the next list gather
   uint32_t commit_pending = 0; // counter slot to clear at the next commit (0: none)
   int32_t *glist, *flist;
-  uint32_t *skey, *srank, *scount, *ccount, *marks, *soff, *spart, *lpre;
+  uint32_t *skey, *srank, *scount, *ccount, *marks, *soff, *spart, *stop, *lpre;
   unsigned long long *lmask;
   void *tmp_state;
   int32_t *tmp_ids;

@@ -48,6 +48,7 @@ SortBuf sort_buf(const aq_sim *s, void *state, int64_t n, int32_t *ids) {
   b.counts = s->scount;
   b.off = s->soff;
   b.part = s->spart;
+  b.top = s->stop;
   b.lmask = s->lmask;
   b.lpre = s->lpre;
   b.item_off = s->item_off;
@@ -75,6 +76,7 @@ int sort_begin(aq_sim *s, hipStream_t st) {
   if (s->sort_open) {
     if ((rc = fill_u32(s->ccount, 0u, s->nodes, st))) return rc;
     if ((rc = fill_u32(s->marks, 0u, s->nblocks, st))) return rc;
+    if ((rc = fill_u32(s->stop, 0u, 2 * (((int64_t)s->nblocks + 64 * kTop - 1) / (64 * kTop)), st))) return rc;
   }
   s->sort_open = true;
   s->have_items = false;

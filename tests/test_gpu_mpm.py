@@ -725,3 +725,12 @@ def test_tiles_at_the_faces_of_the_grid(dim, fluid, n_grid, n):
         got.append(sim.get_state())
     for c in range(got[0].shape[0]):
         assert np.abs(got[0][c] - got[1][c]).max() <= 1e-9 * max(1.0, np.abs(got[1][c]).max()), c
+
+
+@pytest.mark.parametrize("dim, n_grid", [(2, 1024), (2, 1032), (3, 104), (2, 2048)])
+@pytest.mark.parametrize("n", [1, 5000, 60000])
+def test_sort_order_on_large_grids(dim, n_grid, n):
+    """The order of aq_sort at the grid size (16,384 blocks) above which the
+    scan adds up totals of two levels, just above it and at four entries of
+    the upper level."""
+    test_sort_order_layer_by_layer(dim, n_grid, n)
