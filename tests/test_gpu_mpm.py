@@ -734,3 +734,63 @@ def test_sort_order_on_large_grids(dim, n_grid, n):
     scan adds up totals of two levels, just above it and at four entries of
     the upper level."""
     test_sort_order_layer_by_layer(dim, n_grid, n)
+
+
+@pytest.mark.parametrize("dim, n_grid", [(2, 8), (2, 64), (2, 72), (3, 16), (3, 20)])
+@pytest.mark.parametrize("n", [1, 257, 5000])
+def test_sort_order_on_small_grids(dim, n_grid, n):
+    """The order of aq_sort where one workgroup counts and scans all blocks
+    (1 and 64 of them), and just above."""
+    test_sort_order_layer_by_layer(dim, n_grid, n)
+
+
+@pytest.mark.parametrize("dim, fluid, storage", [(2, True, "f32"), (2, False, "f64"), (3, True, "f32"),
+                                                 (3, False, "f64")])
+def test_limits_with_a_nan_particle(dim, fluid, storage):
+    """A particle whose C is NaN, apart from the others, counts for nothing in
+    a range run's limits (folded into the 2D kernels, in a kernel of their own
+    in 3D) nor in those of a single state."""
+    import torch
+    if not torch.cuda.is_available():
+        pytest.skip("no GPU")
+    import autoquantizer_amd as aq
+    print(f"[nan limits] {dim} {fluid} {storage}", flush=True)
+    n, steps = 601, 4
+
+    def make():
+        cfg = aq.MPMConfig()
+        cfg.dim, cfg.use_fluid, cfg.n_grid, cfg.n_particles, cfg.compute_fp = dim, fluid, 32, n, storage
+        cfg.dt, cfg.la, cfg.E, cfg.p_vol = 1e-4, 400.0, 1e3, (0.5 / 32) ** dim
+        sim = aq.MPMSolver(cfg)
+        rng = np.random.default_rng(12)
+        st = np.zeros((sim.ncomp, n))
+        st[:dim] = rng.uniform(0.35, 0.6, (dim, n))
+        st[:dim, 7] = 0.85
+        st[dim:2 * dim] = rng.uniform(-1, 1, (dim, n))
+        st[2 * dim, 7] = np.nan
+        st[-1 if fluid else -dim * dim:] = 1.0 if fluid else np.eye(dim).reshape(-1, 1)
+        sim.set_state(st)
+        return sim
+
+    a = make()
+    a.init_limits()
+    a.advance_detect(steps, sort_every=2)
+    got = a._mxmn.cpu().numpy().reshape(2, -1)
+    mx, mn = np.full(a.ncomp, -np.inf), np.full(a.ncomp, np.inf)
+    for k in range(1, steps + 1):
+        b = make()
+        b.advance(k, sort_every=2)
+        v = b.get_state()
+        assert np.isnan(v).any() and np.isfinite(np.delete(v, 7, axis=1)).all()
+        mx, mn = np.fmax(mx, np.nanmax(v, axis=1)), np.fmin(mn, np.nanmin(v, axis=1))
+    # x moves by 1e-4 a substep; its runs differ by a rounding and 1e-4 of the v's differences.  The others'
+    # sums are taken in another order: 1e-4 (f32) or the limits' own f32 rounding of the component's largest value
+    tol = np.full(a.ncomp, 1e-4 if storage == "f32" else 1e-6)
+    tol[:dim] = 1e-6
+    big = np.maximum(np.abs(mx), np.abs(mn))
+    assert (np.abs(got[0] - mx) <= tol * big).all() and (np.abs(got[1] - mn) <= tol * big).all()
+    b.init_limits()
+    b.detect_bound_kernel()
+    one = b._mxmn.cpu().numpy().reshape(2, -1)
+    np.testing.assert_array_equal(one[0], np.nanmax(v, axis=1).astype(np.float32))
+    np.testing.assert_array_equal(one[1], np.nanmin(v, axis=1).astype(np.float32))
