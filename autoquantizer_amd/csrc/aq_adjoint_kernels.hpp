@@ -183,11 +183,6 @@ __device__ __forceinline__ void adj_sums(const AdjStencil<T> &St, const T (&c)[3
   R.X[0] = ddw(0, qi);
 }
 
-// G2P adjoint of one particle, shared by the tiled and untiled kernels:
-// from its values v (x and J/F used) and the adjoint nx of its next values,
-// the adjoints of x and J/F (xo, jo).  The velocity adjoint of stencil node
-// off, w_n u_n with u_n = vb + 4 inv_dx C_b (off - fx), goes to add(off, w,
-// u); fetch(off) returns the node's velocity.
 // The values are computed here: the compiler may not move their sums down.
 template <class T, int N, int M>
 __device__ __forceinline__ void hold_all(T (&a)[N], T (&b)[M]) {
@@ -197,6 +192,11 @@ __device__ __forceinline__ void hold_all(T (&a)[N], T (&b)[M]) {
   for (int i = 0; i < M; ++i) asm volatile("" : "+v"(b[i]));
 }
 
+// G2P adjoint of one particle, shared by the tiled and untiled kernels:
+// from its stencil, its J/F and the adjoint of its next values (begin), the
+// adjoints of x and J/F (sums: xo, jo).  The velocity adjoint of stencil
+// node off, w_n u_n with u_n = vb + 4 inv_dx C_b (off - fx), goes to add(off,
+// w, u); fetch(off) returns the node's velocity.
 template <int DIM, int MAT, class T> struct AdjG2P {
   using CI = Comps<DIM, MAT>;
   static constexpr int NJF = CI::NC - CI::CJ;
@@ -718,11 +718,11 @@ __global__ void __launch_bounds__(256) k_adj_p2g(const T *__restrict__ st, T *__
 }
 
 // ---- tiled particle phases ---------------------------------------------------
-// Wavefronts per SIMD that registers are kept for (G2P adjoint, P2G adjoint);
-// 3D f64 keeps one.
+// Wavefronts per SIMD that the tiled adjoint kernels' registers are kept for:
+// 3D f64 keeps one (292 to 488 VGPRs).  3D f32 elastic bodies spill 2 (G2P) and
+// 13 (P2G) of 168 VGPRs.
 template <int DIM, class T> struct AdjWaves {
-  static constexpr int G2P = IsF64<T>::value ? (DIM == 3 ? 1 : 2) : (DIM == 3 ? 3 : 4);
-  static constexpr int P2G = IsF64<T>::value ? (DIM == 3 ? 1 : 2) : (DIM == 3 ? 3 : 4);
+  static constexpr int W = IsF64<T>::value ? (DIM == 3 ? 1 : 2) : (DIM == 3 ? 3 : 4);
 };
 
 // G2P adjoint over work items: the velocity tile staged in LDS is read by
@@ -739,7 +739,7 @@ template <int DIM, class T> struct AdjWaves {
 // atomics), of a 3D elastic body 36 and 30; 80,000 of a 2D elastic body, f64:
 // 7.2 both ways (101).
 template <int DIM, int MAT, class T>
-__global__ void __launch_bounds__(kItem) __attribute__((amdgpu_waves_per_eu(AdjWaves<DIM, T>::G2P)))
+__global__ void __launch_bounds__(kItem) __attribute__((amdgpu_waves_per_eu(AdjWaves<DIM, T>::W)))
 k_adj_g2p_tiled(const T *__restrict__ st, const T *__restrict__ adj_next,
                                                          T *__restrict__ adj_out, int64_t cap, int64_t n,
                                                          ParamsT<T> P, const int4 *__restrict__ items,
@@ -858,12 +858,11 @@ k_adj_g2p_tiled(const T *__restrict__ st, const T *__restrict__ adj_next,
 
 // P2G adjoint over work items: the node adjoints staged in LDS, completing
 // adj_out; sum_p adj_out^2 is carried per lane over the workgroup's items
-// and added to gsum once per workgroup; those f64 atomics on one or two
-// cache lines bound the phase (262,144 particles of a 3D fluid, f32: 33 ->
-// 28 us, 15 without sums; 80,000 of a 2D elastic body, f64: 11.7 -> 13 us,
-// 6.5 without sums).
+// and added to gsum once per workgroup by f64 atomics on one or two cache
+// lines (262,144 particles of a 3D fluid, f32: 29 us, 22 without sums; 80,000
+// of a 2D elastic body, f64: 9.6 and 7.2).
 template <int DIM, int MAT, class T>
-__global__ void __launch_bounds__(kItem) __attribute__((amdgpu_waves_per_eu(AdjWaves<DIM, T>::P2G)))
+__global__ void __launch_bounds__(kItem) __attribute__((amdgpu_waves_per_eu(AdjWaves<DIM, T>::W)))
 k_adj_p2g_tiled(const T *__restrict__ st, T *__restrict__ adj_out,
                                                          int64_t cap, int64_t n, ParamsT<T> P,
                                                          const int4 *__restrict__ items,

@@ -102,15 +102,6 @@ template <int DIM> __device__ __forceinline__ void lane_coords(int lane, int (&l
   }
 }
 
-// Gather of P2G results into grid_v, one 64-node block per wavefront.  A
-// node is covered by the tiles of 2^DIM neighbouring blocks (per axis its own
-// block and the one on the side of the block edge it is nearest); each lane
-// reads the item ranges of its 2^DIM blocks and the first two items' tile
-// values all at once (independent loads), then any further items, and sums
-// in a fixed order (neighbour, then item); grid_f is added for blocks flagged by untiled scatters (and zeroed after
-// use).  `emit` takes each node's sum and stores what the caller wants of it.
-// Blocks with no contribution are marked inactive in `act` (and zeroed if
-// they were active).
 // What a gather does with a node's sum: the grid update into grid_v (OP), or
 // the plain (m v, m).
 template <int DIM, class T, bool OP> struct EmitGrid {
@@ -138,7 +129,16 @@ template <class T> struct GatherArgs {
   uint32_t *act;
 };
 
-// Gather of block b (uniform over the wavefront) of one simulation.
+// Gather of P2G results into grid_v: block b (uniform over the wavefront) of
+// one simulation, 64 nodes, one per lane.  A node is covered by the tiles of
+// 2^DIM neighbouring blocks (per axis its own block and the one on the side
+// of the block edge it is nearest); each lane reads the item ranges of its
+// 2^DIM blocks, then the first two items' tile values of four neighbours at
+// a time and their further items one after the other, and sums in a fixed
+// order (neighbour, then item); grid_f is added for blocks flagged by
+// untiled scatters (and zeroed after use).  `emit` takes each node's sum and
+// stores what the caller wants of it.  Blocks with no contribution are
+// marked inactive in `act` (and zeroed if they were active).
 // bm_read (null: every tile whole): per block, bit i set when its item i
 // wrote its tile's drift margin (bit 31: items 31 and later, which always
 // do); the margin nodes of the other items were not written and are not

@@ -107,7 +107,7 @@ struct aq_sim {
   int32_t *tmp_ids;
   int4 *items;
   int32_t *item_off;  // [nblocks + 1]; item_off[nblocks] = item count
-  uint32_t *near;     // [nblocks]: particles within one block (k_near, at each sort)
+  uint32_t *near;     // [nblocks]: particles within one block (sort_scan)
   float *lim_part;    // [kLimSlots][kLimRow]: partial maxima of a range run
   int32_t max_items;
   bool have_items;    // items describe the current order of `items_state`

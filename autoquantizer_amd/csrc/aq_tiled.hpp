@@ -227,16 +227,13 @@ template <> struct AccOf<double> {
   }
 };
 
-template <class T> __device__ __forceinline__ T wave_sum(T x) {
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) x += __shfl_xor(x, o);
-  return x;
-}
-
 // Wavefronts per SIMD that the tiled kernels' registers are kept for: 4
-// (<= 128 VGPRs; the f32 kernels need 83 to 119) except for 3D elastic
-// records with a run-time layout (165 VGPRs; held to 128, the kernel spills
-// thousands of times) and f64 storage (up to 200).
+// (<= 128 VGPRs: the fused kernels of f32 storage need 68 to 114, of records
+// with a run-time layout of up to 16 words 83 to 135) except for 3D elastic
+// records with a run-time layout (161 to 168; held to 128, the kernel spills
+// thousands of times) and f64 storage (102 to 202).  VGPRs spilled: 4 (3D
+// elastic, 16 words) and, grouped, 11 and 4 (3D fluid, 4 and 8 words) and 9
+// (3D elastic, 16 words).
 template <int ST, int DIM, int MAT> struct TiledWaves {
   static constexpr int W = ST == AQ_STORE_F64 ? 2 : (ST == AQ_STORE_QUANT && DIM == 3 && MAT == AQ_ELASTIC ? 3 : 4);
 };
@@ -256,10 +253,11 @@ __device__ __forceinline__ void tile_origin(const int4 &item, int (&o)[3]) {
 // a test, a load and an LDS store.  Blocks outside the grid hold zeros: the
 // item's block lies at some faces of the grid, a node in a neighbour block
 // across some of its own, and the two masks meet if that block is outside.
-// The fused kernel is bound by VALU issue (75 % of its cycles; f32 sums take
-// 2 of them, integer operations and conversions 4), so address arithmetic
-// counts: with the bounds by LaneFold, 32 substeps of 1,048,576 particles of
-// a 3D fluid (32-byte records) took 3.27 ms before and 3.13 ms with this.
+// The fused kernels are bound by VALU issue (a wavefront's f32 sum, product
+// or move takes a SIMD 2.7 cycles, an fma 3.3, a shift, conversion, comparison
+// or integer product 4.4 to 4.8: measured), so address arithmetic counts:
+// with the bounds by LaneFold, 32 substeps of 1,048,576 particles of a 3D
+// fluid (32-byte records) took 3.27 ms before and 3.13 ms with this.
 template <int DIM> struct TileShare {
   using TL = Tile<DIM>;
   static constexpr int R = (TL::TN + kItem - 1) / kItem;  // nodes per thread
@@ -403,10 +401,13 @@ template <int O> __device__ __forceinline__ void half_swap_word(uint32_t &x, uin
 }
 template <int O> __device__ __forceinline__ uint32_t lane_xor_word(uint32_t x) {
   static_assert(O == 8 || O == 4 || O == 2 || O == 1, "");
-  if constexpr (O == 4) return (uint32_t)__builtin_amdgcn_ds_swizzle((int)x, (O << 10) | 31);  // xor mask, 32 lanes
-  // DPP: rotation of a row of 16 by 8; quad permutations [2,3,0,1] and [1,0,3,2]
-  constexpr int ctrl = O == 8 ? 0x128 : (O == 2 ? 0x4E : 0xB1);
-  return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, O == 4 ? 0x128 : ctrl, 0xF, 0xF, true);
+  if constexpr (O == 4) {
+    return (uint32_t)__builtin_amdgcn_ds_swizzle((int)x, (O << 10) | 31);  // xor mask, 32 lanes
+  } else {
+    // DPP: rotation of a row of 16 by 8; quad permutations [2,3,0,1] and [1,0,3,2]
+    constexpr int ctrl = O == 8 ? 0x128 : (O == 2 ? 0x4E : 0xB1);
+    return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, ctrl, 0xF, 0xF, true);
+  }
 }
 template <int O, class E> __device__ __forceinline__ void half_swap(E &x, E &y) {
   constexpr int W = sizeof(E) / 4;
@@ -522,9 +523,6 @@ __device__ __forceinline__ void tiled_run(const Src &src, float *__restrict__ li
   }
   constexpr int NLV = NC <= 16 ? 16 : 32;
   float lmax = -__builtin_inff(), lneg = -__builtin_inff();  // of the lane's component, over the items
-  // one simulation: an item's descriptor is loaded during the item before it
-  // (the particle and tile loads wait for it)
-  int4 next = make_int4(0, 0, 0, 0);
   for (; it < hi; it += per) {
     int li;  // the item's number in its simulation
     const TiledArgs<T> &A = src.args(it, li);
