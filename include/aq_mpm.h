@@ -229,7 +229,8 @@ int aq_g2p(aq_sim *sim, void *state, int64_t n, const int32_t *ids, uint32_t ste
    call's start and then every `sort_every` substeps (0 = never:
    global-memory kernels), so every call with sort_every > 0 costs at least
    one sort: prefer few long calls to many short ones.  ids are permuted
-   along. */
+   along.  If a launch fails, some of the substeps have been done; state and
+   ids are in the same order. */
 int aq_advance(aq_sim *sim, void *state, int64_t n, int nsteps, uint32_t step0,
                int sort_every, int32_t *ids, void *stream);
 
